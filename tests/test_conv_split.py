@@ -67,3 +67,22 @@ def test_padding_is_zero_beside_non_finite_pixels(native):
     assert np.all(np.abs(y - want)[fin] <= bar.reshape(20, 20, 96)[fin])
     big = np.abs(want[9:12, 9:12]) < 3.4e38
     assert np.allclose(y[9:12, 9:12][big], want[9:12, 9:12][big], rtol=1e-5)
+
+
+@pytest.mark.parametrize("H,W,K", [(20, 20, 3), (9, 33, 5)])
+def test_sums_of_elements_that_round_to_zero(native, H, W, K):
+    """Pixels under 2^-134 have no bf16 part: alone in the image (a corner
+    pixel, one that only padded taps reach) and all over it."""
+    announce(f"conv split: subnormal pixels {H}x{W} k{K}")
+    g = rng(H + W)
+    w = g.uniform(500, 1000, (96, K, K, 64)).astype(np.float32)
+    for where in [(0, 0, 0), (0, H - 1, W - 1), (1, 0, W - 1), (1, H - 1, 0), None]:
+        x = np.zeros((2, H, W, 64), np.float32)
+        if where is None:
+            x[:] = g.uniform(2e-41, 4e-41, x.shape)
+        else:
+            x[where] = 3e-41
+        A, B = _im2col(x, K).astype(np.float64), w.reshape(96, -1).T.astype(np.float64)
+        n = K * K * 64
+        err = np.abs(_run(native, x, w) - A @ B)
+        assert np.all(err <= 1e-5 * np.sqrt(n) * (np.abs(A) @ np.abs(B)) + n * 2.0 ** -149), where

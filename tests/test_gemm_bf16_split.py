@@ -124,6 +124,48 @@ def test_extreme_magnitudes(native, tile, name, a, b):
     assert np.all(np.abs(C - A64 @ B64) <= bar)
 
 
+def _near_the_bottom(C, A, B):
+    A64, B64 = A.astype(np.float64), B.astype(np.float64)
+    K = A.shape[1]
+    bar = 1e-5 * np.sqrt(K) * (np.abs(A64) @ np.abs(B64)) + K * 2.0 ** -149
+    return np.all(np.abs(C - A64 @ B64) <= bar)
+
+
+@pytest.mark.parametrize("tile", [1, 5])
+@pytest.mark.parametrize("a,b,K", [(4e-41, 1e3, 8192), (1e-41, 1.0, 8192), (4e-41, 1e3, 70),
+                                   (1e-44, 900.0, 333), (1e-30, 1e-9, 2048)])
+def test_sums_of_elements_that_round_to_zero(native, tile, a, b, K):
+    """|x| under 2^-134 has no bf16 part, and a product under 2^-149 no value:
+    the sums of many are normal floats."""
+    announce(f"bf16 split tile {tile}: {a} by {b}, K={K}")
+    g = rng(K)
+    A = (np.float64(a) * g.uniform(0.5, 1, (140, K))).astype(np.float32)
+    B = (np.float64(b) * g.uniform(0.5, 1, (K, 135))).astype(np.float32)
+    B[:, 7] = 0.0
+    assert _near_the_bottom(_run(native, A, B, tile=tile), A, B)
+
+
+@pytest.mark.parametrize("tile", [1, 5])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_one_subnormal_element_anywhere(native, tile, ta, tb):
+    """A single element that rounds to zero beside zeros, at the edges of the
+    tiles and of the K range, in A or in B: its row (column) is not lost."""
+    M, N, K = 259, 133, 277
+    for r, k in [(0, 0), (258, 276), (127, 255), (128, 256), (255, 16), (256, 275), (31, 1)]:
+        announce(f"bf16 split tile {tile} ta={ta} tb={tb}: subnormal at {r}, {k}")
+        for swap in (False, True):
+            g = rng(r + k)
+            A, B = np.zeros((M, K), np.float32), np.zeros((K, N), np.float32)
+            small, big = (B.T, A.T) if swap else (A, B)
+            r_ = min(r, small.shape[0] - 1)
+            small[r_, k] = 3e-41
+            big[:] = g.uniform(1000, 1023, big.shape)
+            C = _run(native, np.ascontiguousarray(A.T) if ta else A,
+                     np.ascontiguousarray(B.T) if tb else B, ta, tb, tile,
+                     splits=2 if swap else 1)
+            assert _near_the_bottom(C, A, B), (r, k, swap)
+
+
 @pytest.mark.parametrize("tile", [1, 5])
 def test_rows_of_any_scale_keep_their_accuracy(native, tile):
     """Rows of A and columns of B from 1e-12 to 1e12, elements over 1e16 within
