@@ -167,6 +167,23 @@ def test_one_subnormal_element_anywhere(native, tile, ta, tb):
 
 
 @pytest.mark.parametrize("tile", [1, 5])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(33, 65, 1), (257, 129, 5), (130, 131, 8), (259, 70, 71),
+                                   (128, 257, 130)])
+def test_products_redone_whole(native, tile, ta, tb, M, N, K):
+    """Every sum small beside elements that lose parts: all of C comes from
+    the fp32 matrix cores."""
+    announce(f"bf16 split tile {tile} redone {M}x{N}x{K} ta={ta} tb={tb}")
+    g = rng(M + N + K)
+    A = (1e-34 * g.normal(0, 1, (M, K))).astype(np.float32)
+    B = g.normal(0, 1, (K, N)).astype(np.float32)
+    for splits in (1, 2) if K >= 64 else (1,):
+        C = _run(native, np.ascontiguousarray(A.T) if ta else A,
+                 np.ascontiguousarray(B.T) if tb else B, ta, tb, tile, splits, pad=3, off=1)
+        assert _near_the_bottom(C, A, B)
+
+
+@pytest.mark.parametrize("tile", [1, 5])
 def test_rows_of_any_scale_keep_their_accuracy(native, tile):
     """Rows of A and columns of B from 1e-12 to 1e12, elements over 1e16 within
     a row: every element within the bar of its own sum |a b|."""
