@@ -30,8 +30,11 @@
 // 21.0 stay.  (One after the other, in a run of its own: 76.8 -> 64.9, 40.8 ->
 // 37.3, 199 -> 132, 515 -> 366, 56.4 -> 60.9.)  Error against float64 5.1e-7 ->
 // 4.1e-7 at 1000 keys.
-// Non-finite results and results so small that parts below bf16's normal range
-// could show are redone by the wave on the fp32 matrix cores (redo below).
+// Non-finite scores and results so small that parts below bf16's subnormals
+// could show are redone by the two waves of the row group on the fp32 matrix
+// cores (below).  24x1000x1000, us: 46; a NaN in V, or a zero column beside large
+// ones, 48; every row redone 145 (543 with one wave and 4-byte loads; 70 on
+// attention_k).
 #pragma once
 
 #include "bf16_split.h"
@@ -136,7 +139,8 @@ void attention_split_k(attn_args a) {
   using C = sa_cfg<D>;
   constexpr int NB = D / 32;  // 32-wide blocks of O
   __shared__ uint4 lds[2 * C::kBuf];
-  __shared__ float smx[2][kSaWaves];
+  __shared__ float smx[2][kSaWaves], smv[kSaWaves][kWave];
+  __shared__ int sbad[4];
   const int t = threadIdx.x, lane = t % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
   const int c = lane % 32, s = lane / 32;
@@ -386,6 +390,7 @@ void attention_split_k(attn_args a) {
   block(std::false_type{}, nblocks - 1);
 
   // Merge the key halves through LDS: half 1 parks (O, m, l), half 0 combines.
+  smv[wave][lane] = mv;  // t % D = lane: the largest |V| of column `lane`
   {
     const float q = wave_max(mqk), v = wave_max(mv);
     if (lane == 0) {
@@ -396,92 +401,119 @@ void attention_split_k(attn_args a) {
   float *X = reinterpret_cast<float *>(lds) + rg * (16 * NB + 2) * kWave;
   // K's slots: the last block reads only V's.
   static_assert(4 * (16 * NB + 2) * kWave <= 2 * C::kKs * 4, "merge area");
-  if (kh == 1) {
+  auto park = [&] {
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) X[(16 * j + r) * kWave + lane] = acc[j][r];
     X[(16 * NB) * kWave + lane] = sm.m;
     X[(16 * NB + 1) * kWave + lane] = sm.l;
-  }
-  __syncthreads();
-  if (kh == 1) return;
-  float lt;
-  float bq = 1.0f, bv = 1.0f;
-#pragma unroll
-  for (int w = 0; w < kSaWaves; ++w) {
-    bq = fmaxf(bq, smx[0][w]);
-    bv = fmaxf(bv, smx[1][w]);
-  }
-  // Sums the split cannot vouch for (as in sgemm_split_k): non-finite ones;
-  // nonzero ones under thr, and zeros beside values over 1024; and scores of
-  // operands over 2^60, where what a part below the normal range loses could
-  // move a score.
-  const float thr = bv * float(Sk) * 0x1p-99f;
-  bool bad = bq > 0x1p60f;
-  {
+  };
+  float lt = 0.0f, mm = 0.0f;
+  auto merge = [&] {
     const float m1 = X[(16 * NB) * kWave + lane], l1 = X[(16 * NB + 1) * kWave + lane];
-    const float mm = fmaxf(sm.m, m1);
+    mm = fmaxf(sm.m, m1);
     const float e0 = mm == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(sm.m - mm);
     const float e1 = mm == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - mm);
     lt = sm.l * e0 + l1 * e1;
-    bad = bad || !(lt < INFINITY) || !(mm < INFINITY);
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        acc[j][r] = acc[j][r] * e0 + X[(16 * j + r) * kWave + lane] * e1;
+  };
+  if (kh == 1) park();
+  __syncthreads();
+  if (kh == 0) {
+    merge();
+    float bq = 1.0f, bv = 1.0f;
+#pragma unroll
+    for (int w = 0; w < kSaWaves; ++w) {
+      bq = fmaxf(bq, smx[0][w]);
+      bv = fmaxf(bv, smx[1][w]);
+    }
+    // What the split cannot vouch for (s3_check in gemm_split.h has the bounds):
+    // scores of operands over 2^60, where what an element under 2^-110 loses
+    // could move a score; rows whose maximum or sum is not finite; and in O,
+    // before the division,
+    //   - small values: P loses at most 2^-134 an element, V too if under 2^-110,
+    //     Sk (1 + max |V|) 2^-134 in a column of V, and nothing if that is zero;
+    //   - non-finite ones, unless V leaves no way to them but a NaN element.
+    bool bad = bq > 0x1p60f || !(lt < INFINITY) || !(mm < INFINITY);
+    const float sk = float(Sk), thr = sk * bv * 0x1p-108f;
+    uint32_t lo = 0xffffffffu;
+    float nf = 0.0f;
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float o = acc[j][r] * e0 + X[(16 * j + r) * kWave + lane] * e1;
-        const float mag = fabsf(o);
-        bad = bad || !(mag < INFINITY) || (mag < thr && (mag != 0.0f || bv > 1024.0f));
-        acc[j][r] = o;
+        nf = fmaf(acc[j][r], 0.0f, nf);
+        lo = min(lo, __float_as_uint(acc[j][r]) << 1);
       }
-  }
-  if (__any(bad)) {
-    // The wave's rows once more on the fp32 matrix cores (32x32x2: lane (c, s)
-    // supplies k slot s), straight from memory, the key halves one after the
-    // other, a few times slower.
-    sa_row h0;
-    floatx16 acc0[NB];
+    if (__builtin_expect(__any(nf != 0.0f || lo < __float_as_uint(thr) << 1), 0)) {
+      bad = bad || (nf != 0.0f && !(bv < 0x1p127f && sk * bv < 0x1p126f));
 #pragma unroll
-    for (int j = 0; j < NB; ++j) acc[j] = zero16();
-#pragma unroll 1
-    for (int h = 0; h < 2; ++h) {
-      h0 = sm;
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int d = 32 * j + 8 * (r / 4) + 4 * s + r % 4;
+          float cv = 0.0f;
+#pragma unroll
+          for (int w = 0; w < kSaWaves; ++w) cv = fmaxf(cv, smv[w][d]);
+          bad = bad || (cv > 0.0f && fabsf(acc[j][r]) < sk * fmaxf(cv, 1.0f) * 0x1p-108f);
+        }
+    }
+    bad = __any(bad);
+    if (lane == 0) sbad[rg] = bad;
+  }
+  __syncthreads();
+  if (__builtin_expect(sbad[0] | sbad[1] | sbad[2] | sbad[3], 0)) {  // the whole workgroup
+    // The flagged row groups once more on the fp32 matrix cores (32x32x2: lane
+    // (c, s) supplies k slot s), straight from memory, each wave its key half.
+    // Slot s of step e takes d 8 g + 4 s + e, so Q and K come 16 bytes a lane.
+    if (sbad[rg]) {
       sm = sa_row{};
 #pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        acc0[j] = acc[j];
-        acc[j] = zero16();
-      }
-      for (int key0 = 32 * h; key0 < Sk; key0 += 64) {
-        floatx16 st = zero16();
-        const float *kp = K + int64_t(min(key0 + c, Sk - 1)) * a.ldk;
-#pragma unroll 4
-        for (int d = 0; d < D; d += 2)
-          st = __builtin_amdgcn_mfma_f32_32x32x2f32(kp[d + s], qrow[d + s], st, 0, 0, 0);
-        const float alpha = sm.step(st, scale2, key0, s, Sk);
+      for (int j = 0; j < NB; ++j) acc[j] = zero16();
+      f4u q[D / 8];
 #pragma unroll
-        for (int j = 0; j < NB; ++j) acc[j] *= alpha;
+      for (int g = 0; g < D / 8; ++g)
+        q[g] = *reinterpret_cast<const f4u *>(qrow + 8 * g + 4 * s);
+#pragma unroll 1
+      for (int key0 = 32 * kh; key0 < Sk; key0 += kSaKeys) {
+        const float *kp = K + int64_t(min(key0 + c, Sk - 1)) * a.ldk + 4 * s;
+        f4u k4[D / 8];
+#pragma unroll
+        for (int g = 0; g < D / 8; ++g) k4[g] = *reinterpret_cast<const f4u *>(kp + 8 * g);
+        float v[16][NB];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int key = key0 + 8 * (r / 4) + 4 * s + r % 4;
           const float *vp = V + int64_t(min(key, Sk - 1)) * a.ldv + c;
 #pragma unroll
-          for (int j = 0; j < NB; ++j)
-            acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(key < Sk ? vp[32 * j] : 0.0f, st[r],
-                                                          acc[j], 0, 0, 0);
+          for (int j = 0; j < NB; ++j) v[r][j] = key < Sk ? vp[32 * j] : 0.0f;
         }
+        floatx16 sc = zero16();
+#pragma unroll
+        for (int g = 0; g < D / 8; ++g)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(k4[g][e], q[g][e], sc, 0, 0, 0);
+        const float alpha = sm.step(sc, scale2, key0, s, Sk);
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[j] *= alpha;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+#pragma unroll
+          for (int j = 0; j < NB; ++j)
+            acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[r][j], sc[r], acc[j], 0, 0, 0);
       }
+      if (kh == 1) park();
     }
-    const float mm = fmaxf(h0.m, sm.m);
-    const float e0 = mm == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(h0.m - mm);
-    const float e1 = mm == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(sm.m - mm);
-    lt = h0.l * e0 + sm.l * e1;
-#pragma unroll
-    for (int j = 0; j < NB; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[j][r] = acc0[j][r] * e0 + acc[j][r] * e1;
+    __syncthreads();
+    if (kh == 0 && sbad[rg]) merge();
   }
+  if (kh == 1) return;
   if (row >= Sq) return;
   const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
   // Register r of block j is O[row][32 j + 8 (r / 4) + 4 s + r % 4].

@@ -128,3 +128,39 @@ def test_extreme_magnitudes(native, qs, vs):
     top = np.abs(V).max(1, keepdims=True).astype(np.float64)
     assert np.all(np.isfinite(O))
     assert np.all(np.abs(O - want) <= factor * np.maximum(mag, top * (factor > 1e-3)) + 1e-44)
+
+
+@pytest.mark.parametrize("Sq,Sk", [(128, 576), (97, 530), (130, 31 + 512)])
+def test_values_near_the_bottom_of_the_range(native, Sq, Sk):
+    """V elements under 2^-134 have no bf16 part; their averages are not zero.
+    Beside columns of zeros, and in one head of many.  Each of the Sk products
+    of P and V rounds to a subnormal once: Sk * 2^-149 above the bar."""
+    announce(f"attention split: subnormal values {Sq} x {Sk}")
+    g = rng(Sq + Sk)
+    b = 200
+    Q, K, V = (g.normal(0, 1, (b, s, D)).astype(np.float32) for s in (Sq, Sk, Sk))
+    V[3] = g.uniform(2e-41, 4e-41, V[3].shape)
+    V[3, :, 7] = 0.0
+    V[7] = (1e-36 * V[7]).astype(np.float32)
+    V[9, :, 5], V[9, :, 6] = 0.0, 2000.0 * V[9, :, 6]
+    O = _run(native, Q, K, V, 0.125)
+    want, mag = _ref(Q, K, V, 0.125)
+    assert np.all(np.abs(O - want) <= 2e-5 * mag + Sk * 2.0 ** -149)
+    assert np.all(O[3, :, 7] == 0.0) and np.all(O[9, :, 5] == 0.0)
+
+
+@pytest.mark.parametrize("Sq,Sk", [(128, 576), (97, 530), (130, 31 + 512)])
+def test_rows_redone(native, Sq, Sk):
+    """An infinite value in some heads: their rows come from the fp32 matrix
+    cores, and agree in every other column; a NaN stays in its column."""
+    announce(f"attention split: rows redone {Sq} x {Sk}")
+    g = rng(Sq + Sk)
+    b = 200
+    Q, K, V = (g.normal(0, 1, (b, s, D)).astype(np.float32) for s in (Sq, Sk, Sk))
+    want, mag = _ref(Q, K, V, 0.125)
+    V[::3, Sk - 1, 63], V[1::3, 0, 2] = np.inf, np.nan
+    O = _run(native, Q, K, V, 0.125)
+    assert np.all(np.isposinf(O[::3, :, 63])) and np.all(np.isnan(O[1::3, :, 2]))
+    same = np.ones(O.shape, bool)
+    same[::3, :, 63] = same[1::3, :, 2] = False
+    assert np.all((np.abs(O - want) <= 2e-5 * mag)[same])
