@@ -11,6 +11,7 @@
 #include <string>
 
 #include "../../include/silgpu.h"
+#include "intmath.h"
 
 namespace silgpu {
 
@@ -198,8 +199,6 @@ inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 
 __device__ __forceinline__ bool aligned16_dev(const void *p) {
   return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }
-
-inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // ---- device helpers ---------------------------------------------------------
 

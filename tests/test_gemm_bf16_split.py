@@ -229,3 +229,29 @@ def test_large_c_and_a_row_stride_past_the_lane_offsets(native):
     for tile in (TILE_128x128, TILE_256x128):
         native.sgemm_tuned(0, 0, M, N, K, buf, ld, 0, dB, N, 0, dC, N, 0, tile=tile, splits=1)
         _check(down(native, dC, (M, N)), A[:M, :K].copy(), B[:K, :N].copy())
+
+
+@pytest.mark.parametrize("M,N,K,ta,tb,fp32_splits", [
+    (1675, 1882, 4787, 0, 0, 4), (3776, 2496, 4096, 0, 1, 8), (1472, 2560, 2048, 0, 0, 4),
+    (2496, 1984, 6784, 1, 0, 16), (768, 3072, 2048, 1, 0, 4), (301, 2510, 2363, 0, 0, 6),
+    (2368, 1344, 2560, 0, 0, 4)])
+def test_planned_products_are_no_less_accurate(native, M, N, K, ta, tb, fp32_splits):
+    """The library's own plan against the fp32 matrix cores with the K splits
+    that a plan on fp32 tiles alone has: error over 256 rows of C.  The two
+    errors are sums of 256 N independent roundings, so their ratio is known to
+    about 2 / sqrt(256 N) < 0.4%."""
+    announce(f"planned accuracy {M}x{N}x{K} ta={ta} tb={tb}")
+    g = rng(M + K)
+    A = g.uniform(-1, 1, (K, M) if ta else (M, K)).astype(np.float32)
+    B = g.uniform(-1, 1, (N, K) if tb else (K, N)).astype(np.float32)
+    rows = np.sort(g.choice(M, 256, replace=False))
+    want = (A[:, rows].T if ta else A[rows]).astype(np.float64) @ (B.T if tb else B).astype(
+        np.float64)
+    dA, dB, dC = up(native, A), up(native, B), empty(native, M * N)
+    lda, ldb = (M if ta else K), (K if tb else N)
+    native.sgemm(ta, tb, M, N, K, dA, lda, 0, dB, ldb, 0, dC, N, 0)
+    err = np.linalg.norm(down(native, dC, (M, N))[rows] - want)
+    native.sgemm_tuned(ta, tb, M, N, K, dA, lda, 0, dB, ldb, 0, dC, N, 0, tile=2,
+                       splits=fp32_splits)
+    fp32 = np.linalg.norm(down(native, dC, (M, N))[rows] - want)
+    assert err <= 1.004 * fp32, (err / fp32, native.last_plan())
