@@ -98,6 +98,13 @@ inline bool split_range_ok(double range, double fp32_range) {
   return range * (t[i - 1].r2 + f * (t[i].r2 - t[i - 1].r2)) <= fp32_range;
 }
 
+// K splits that the fp32 plan would not have needed take at most this much for
+// their partial planes.
+constexpr double kMaxPlaneBytes = 0x1p30;
+inline double plane_bytes(int sp, int64_t M, int64_t N) {
+  return sp > 1 ? double(sp) * double(M) * double(N) * 4.0 : 0.0;
+}
+
 inline double plane_sum_time(int sp, int64_t rows, int64_t cols) {
   return 0.8e-6 + double(sp + 1) * double(rows) * double(cols) * 4.0 / 5.0e12 + 0.05e-6 * sp;
 }
@@ -183,6 +190,9 @@ inline fp32_pick fp32_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool 
       // (3- and 6-way splits of the larger tiles won nowhere in the sweeps.)
       if ((sp == 3 || sp == 6) && wide) continue;
       if (!short_enough(plan{cd.tile, sp})) continue;
+      if (max_range > 0.0 && double(sp) * max_range > double(K) * 1.001 &&
+          plane_bytes(sp, M, N) > kMaxPlaneBytes)
+        continue;  // more K splits than accuracy asks for
       const int64_t wg = tiles(cd.bm, cd.bn) * sp;
       const double klen = double(cdiv(cdiv(K, sp), cd.bk) * cd.bk);
       double t = round_time(cd, wg, klen);
@@ -296,8 +306,13 @@ inline plan choose_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool dtl
   const fp32_pick ref = fp32_plan(M, N, K, batch, dtl_ok, 0.0);
   const double range = k_range(ref.p, M, K);
   fp32_pick pick = ref;
-  if (ref.p.tile == TILE_256x256 || ref.p.tile == TILE_128x128)
+  int min_splits = (2 * ref.p.splits + 2) / 3;
+  if (ref.p.tile == TILE_256x256 || ref.p.tile == TILE_128x128) {
     pick = fp32_plan(M, N, K, batch, dtl_ok, range);
+    // On the bf16 tiles also no fewer than two thirds of the K splits that suit
+    // the tiles that run best.
+    min_splits = (2 * fp32_plan(M, N, K, batch, dtl_ok, INFINITY).p.splits + 2) / 3;
+  }
   if (pick.time == 0.0) return pick.p;  // by rule
   plan best = pick.p;
   // The bf16 kernel's tiles (gemm_split.h), one workgroup per CU: `launch`
@@ -315,13 +330,12 @@ inline plan choose_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool dtl
   // loads, which the model leaves out, and the bf16 kernel nothing.
   double to_beat = pick.time * (vec ? 0.90 : 1.15);
   for (const wide_cand &w : wides) {
-    for (int sp : {1, 2, 3, 4, 5, 6, 8, 12, 16}) {
+    for (int sp : {1, 2, 3, 4, 6, 8, 12, 16}) {
       if (batch != 1 ? sp > 1 || K < 320 : sp > 1 && K / sp < 128) continue;
-      if (!split_range_ok(double(K) / sp, range)) continue;
-      // (5 and 16 splits are there for accuracy alone.)
-      if (sp == 5 && split_range_ok(double(K) / 4, range)) continue;
+      if (!split_range_ok(double(K) / sp, range) || sp < min_splits) continue;
+      // (16 splits are there for accuracy alone.)
       if (sp == 16 && split_range_ok(double(K) / 12, range)) continue;
-      if (batch == 1 && K > 8192 * int64_t(sp) && sp < 12) continue;
+      if (sp > ref.p.splits && plane_bytes(sp, M, N) > kMaxPlaneBytes) continue;
       const int64_t wg = tiles(w.bm, w.bn) * sp;
       const double stages =
           double(cdiv(cdiv(K, sp), w.bk)) + (K % w.bk ? 1.5 : 0.0);

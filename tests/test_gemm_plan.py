@@ -115,3 +115,15 @@ def test_no_plan_adds_up_more_in_a_row_than_the_fp32_tiles_would(plans):
     assert sum(_bf16(p) for p, _ in got) > 3000
     for (M, N, K, b, _), (p, f) in zip(shapes, got):
         assert _worse(p, f, M, K) <= 1.005, ((M, N, K, b), p, f)
+
+
+def test_large_products_need_no_workspace_that_they_never_needed(plans):
+    """Partial planes stay within 1 GiB where the fp32 tiles' plan has none."""
+    rng = random.Random(2)
+    shapes = [(n, n, n, 1, True) for n in (8192, 16384, 32768, 65536, 70000, 100000)]
+    shapes += [(*_draw(rng, 120000), 1, True) for _ in range(5000)]
+    got = plans(shapes)
+    assert all(p[1] == 1 for p, _ in got[:6])
+    for (M, N, K, _, _), (p, f) in zip(shapes, got):
+        planes = 4.0 * M * N * p[1] if p[1] > 1 else 0.0
+        assert planes <= max(2.0 ** 30, 4.0 * M * N * f[1] if f[1] > 1 else 0.0), (M, N, K, p, f)
