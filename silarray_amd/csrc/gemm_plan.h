@@ -314,7 +314,6 @@ inline plan choose_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool dtl
     min_splits = (2 * fp32_plan(M, N, K, batch, dtl_ok, INFINITY).p.splits + 2) / 3;
   }
   if (pick.time == 0.0) return pick.p;  // by rule
-  plan best = pick.p;
   // The bf16 kernel's tiles (gemm_split.h), one workgroup per CU: `launch`
   // once, per round of workgroups `fixed` for the first loads and the stores
   // and per K tile c0 with an idle chip around it, c1 more with every CU busy;
@@ -326,36 +325,41 @@ inline plan choose_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool dtl
   };
   const wide_cand wides[] = {{TILE_256x256, 256, 128, 16, 0.92e-6, 0.28e-6, 5.5e-6, 5.0e-6},
                              {TILE_128x128, 128, 128, 32, 1.13e-6, 0.27e-6, 3.5e-6, 4.0e-6}};
-  // Rows that are not 16-byte aligned cost the register-staged tiles scalar
-  // loads, which the model leaves out, and the bf16 kernel nothing.
-  double to_beat = pick.time * (vec ? 0.90 : 1.15);
-  for (const wide_cand &w : wides) {
-    for (int sp : {1, 2, 3, 4, 6, 8, 12, 16}) {
-      if (batch != 1 ? sp > 1 || K < 320 : sp > 1 && K / sp < 128) continue;
-      if (!split_range_ok(double(K) / sp, range) || sp < min_splits) continue;
-      // (16 splits are there for accuracy alone.)
-      if (sp == 16 && split_range_ok(double(K) / 12, range)) continue;
-      if (sp > ref.p.splits && plane_bytes(sp, M, N) > kMaxPlaneBytes) continue;
-      const int64_t wg = tiles(w.bm, w.bn) * sp;
-      const double stages =
-          double(cdiv(cdiv(K, sp), w.bk)) + (K % w.bk ? 1.5 : 0.0);
-      double t = w.launch + double(cdiv(wg, 256)) *
-                                (w.fixed + stages * (w.c0 + w.c1 * (wg < 256 ? double(wg) / 256.0
-                                                                              : 1.0)));
-      if (sp > 1) t += plane_sum_time(sp, M, N);
-      if (t < to_beat) {
-        to_beat = t;
-        best = plan{w.tile, sp};
-        if (w.tile == TILE_256x256 && M * N >= kWideC) {
-          best.tile = TILE_128x64;
-          best.wide = true;
+  // The pick by time; where it sums too long a range, the pick among those that
+  // do not, with 5 and 16 splits as well.
+  for (const bool exact : {false, true}) {
+    // Rows that are not 16-byte aligned cost the register-staged tiles scalar
+    // loads, which the model leaves out, and the bf16 kernel nothing.
+    double to_beat = pick.time * (vec ? 0.90 : 1.15);
+    plan best = pick.p;
+    bool wide = false;
+    for (const wide_cand &w : wides) {
+      for (int sp : {1, 2, 3, 4, 5, 6, 8, 12, 16}) {
+        if (batch != 1 ? sp > 1 || K < 320 : sp > 1 && K / sp < 128) continue;
+        if (!exact && (sp == 5 || sp == 16)) continue;
+        if (sp < min_splits || (exact && !split_range_ok(double(K) / sp, range))) continue;
+        if (sp > ref.p.splits && plane_bytes(sp, M, N) > kMaxPlaneBytes) continue;
+        const int64_t wg = tiles(w.bm, w.bn) * sp;
+        const double stages = double(cdiv(cdiv(K, sp), w.bk)) + (K % w.bk ? 1.5 : 0.0);
+        const double fill = wg < 256 ? double(wg) / 256.0 : 1.0;
+        double t = w.launch +
+                   double(cdiv(wg, 256)) * (w.fixed + stages * (w.c0 + w.c1 * fill));
+        if (sp > 1) t += plane_sum_time(sp, M, N);
+        if (t < to_beat) {
+          to_beat = t;
+          wide = true;
+          best = plan{w.tile, sp};
+          if (w.tile == TILE_256x256 && M * N >= kWideC) {
+            best.tile = TILE_128x64;
+            best.wide = true;
+          }
         }
       }
     }
+    if (!wide || exact || split_range_ok(double(K) / best.splits, range)) return best;
   }
-  return best;
+  return pick.p;
 }
-
 
 }  // namespace
 }  // namespace silgpu
