@@ -284,9 +284,9 @@ int silgpu_sgemm(int trans_a, int trans_b, int64_t M, int64_t N, int64_t K,
 
 /* silgpu_sgemm with a forced kernel configuration, for tile sweeps.  No
  * reference counterpart.  tile: 1 = 128x128, 2 = 64x64, 3 = 32x128,
- * 4 = 128x64, 5 = 256x256 (tile of C; 1 and 5, and 4 where C has at least
- * 1.5 * 2^20 elements, run on the bf16 matrix cores with every float split
- * exactly in three, 5 and such a 4 as 256x128 workgroups); 6, 7, 8 = the small-M
+ * 4 = 128x64, 5 = 256x256 (tile of C; 1 and 5 run on the bf16 matrix cores
+ * with every float split exactly in three, 5 as 256x128 workgroups, and where a
+ * row stride along K is 2^21 floats or more as 4); 6, 7, 8 = the small-M
  * kernel (M <= 32, batch 1, A not transposed; otherwise the 32x128 tile)
  * with 32, 64 or 128 columns per workgroup; 9 = 64x64 with each
  * workgroup's K range halved between two groups of waves (M, N, K

@@ -11,8 +11,8 @@
 namespace silgpu {
 namespace {
 
-// Tile configurations.  128x128 and 256x256 run on the bf16 kernel, as 128 x
-// 128 and 256 x 128 workgroups.
+// Tile configurations.  128x128 and 256x256 run on the bf16 kernel
+// (gemm_split.h), as 128 x 128 and 256 x 128 workgroups; each id names one kernel.
 enum tile_cfg {
   TILE_AUTO = 0,
   TILE_128x128 = 1,
@@ -32,10 +32,6 @@ enum tile_cfg {
   TILE_64x64_K4 = 10
 };
 
-// Elements of C from which TILE_128x64, forced, runs as 256 x 128 workgroups
-// of the bf16 kernel.  (By plan it does where the model says so.)
-constexpr int64_t kWideC = int64_t(3) << 19;
-
 struct plan {
   int tile;
   int splits;
@@ -43,8 +39,6 @@ struct plan {
   // tail_splits K splits (the main product then fills whole rounds of CUs).
   int tail_rows = 0;
   int tail_splits = 1;
-  // TILE_128x64 as 256 x 128 workgroups of the bf16 kernel (gemm_split.h).
-  bool wide = false;
 };
 
 // The 32x128 tile for M <= 32, K split for about 256 workgroups.
@@ -349,10 +343,6 @@ inline plan choose_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool dtl
           to_beat = t;
           wide = true;
           best = plan{w.tile, sp};
-          if (w.tile == TILE_256x256 && M * N >= kWideC) {
-            best.tile = TILE_128x64;
-            best.wide = true;
-          }
         }
       }
     }

@@ -1,5 +1,5 @@
 """The products that run on the bf16 matrix cores with every float split in
-three (forced tiles 1 and 5, and 4 on a large C), against float64.
+three (forced tiles 1 and 5), against float64.
 
 Bars: the SGEMM bar of gpu_util (1e-5 sqrt(K) of sum |a b| per element and
 normwise); the split itself stays under it by far (2^-26 per product).  Sums
@@ -210,16 +210,27 @@ def test_no_less_accurate_than_the_fp32_instruction(native, K):
     assert err[1] <= err[2] and err[5] <= err[2], err
 
 
-def test_large_c_and_a_row_stride_past_the_lane_offsets(native):
-    """Tile 4 on a C of 1.5 M elements runs the 256 x 128 workgroups; a
-    K-contiguous operand with rows 2^21 floats apart takes other tiles."""
-    announce("bf16 split: wide tile 4, long rows")
+def test_each_tile_id_names_one_kernel(native):
+    """Tile 4 stays the fp32 128 x 64 tile on a C of 1.5 M elements and beyond, tile
+    5 the bf16 kernel, and the plan that silgpu_gemm_last_plan reports gives the
+    same bits when forced; a K-contiguous operand with rows 2^21 floats apart
+    takes the fp32 tiles."""
+    announce("bf16 split: tile ids, long rows")
     g = rng(4)
-    A = g.normal(0, 1, (2048, 40)).astype(np.float32)
-    B = g.normal(0, 1, (40, 768)).astype(np.float32)
+    A = g.normal(0, 1, (2048, 3072)).astype(np.float32)
+    B = g.normal(0, 1, (3072, 768)).astype(np.float32)
     C4 = _run(native, A, B, tile=TILE_128x64)
-    assert np.array_equal(C4, _run(native, A, B, tile=TILE_256x128))
+    assert native.last_plan() == [(TILE_128x64, 1, 2048)]
+    C5 = _run(native, A, B, tile=TILE_256x128)
+    assert native.last_plan() == [(TILE_256x128, 1, 2048)]
+    assert not np.array_equal(C4, C5)  # other instructions, other roundings
     _check(C4, A, B)
+    dA, dB, dC = up(native, A), up(native, B), empty(native, 2048 * 768)
+    native.sgemm(0, 0, 2048, 768, 3072, dA, 3072, 0, dB, 768, 0, dC, 768, 0)
+    (tile, splits, rows), = native.last_plan()
+    assert rows == 2048
+    want = down(native, dC, (2048, 768))
+    assert np.array_equal(_run(native, A, B, tile=tile, splits=splits), want)
     M, N, K, ld = 5, 150, 33, 1 << 21
     buf = empty(native, M * ld)
     for m in range(M):
@@ -228,6 +239,7 @@ def test_large_c_and_a_row_stride_past_the_lane_offsets(native):
     dB, dC = up(native, np.ascontiguousarray(B[:K, :N])), empty(native, M * N)
     for tile in (TILE_128x128, TILE_256x128):
         native.sgemm_tuned(0, 0, M, N, K, buf, ld, 0, dB, N, 0, dC, N, 0, tile=tile, splits=1)
+        assert native.last_plan() == [(TILE_128x64, 1, M)]
         _check(down(native, dC, (M, N)), A[:M, :K].copy(), B[:K, :N].copy())
 
 

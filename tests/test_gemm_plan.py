@@ -26,8 +26,8 @@ int main() {
   while (std::scanf("%lld %lld %lld %lld %d %d", &M, &N, &K, &batch, &dtl, &vec) == 6) {
     const plan p = choose_plan(M, N, K, batch, dtl, vec);
     const plan f = fp32_plan(M, N, K, batch, dtl, 0.0).p;
-    std::printf("%d %d %d %d %d  %d %d %d %d\n", p.tile, p.splits, p.tail_rows, p.tail_splits,
-                int(p.wide), f.tile, f.splits, f.tail_rows, f.tail_splits);
+    std::printf("%d %d %d %d  %d %d %d %d\n", p.tile, p.splits, p.tail_rows, p.tail_splits,
+                f.tile, f.splits, f.tail_rows, f.tail_splits);
   }
 }
 """
@@ -48,13 +48,13 @@ def plans(tmp_path_factory):
         out = subprocess.run([str(d / "driver")], input=text, check=True, capture_output=True,
                              text=True).stdout.split("\n")
         rows = [tuple(map(int, line.split())) for line in out if line]
-        return [(r[:5], r[5:]) for r in rows]
+        return [(r[:4], r[4:]) for r in rows]
 
     return run
 
 
 def _bf16(p):
-    return p[0] in (TILE_128x128, TILE_256x128) or p[4]
+    return p[0] in (TILE_128x128, TILE_256x128)
 
 
 def _squared_error(tile, splits, tail_rows, tail_splits, M, K):
@@ -72,7 +72,7 @@ MEASURED = [(256, 0.69), (768, 0.728), (2048, 0.748), (8192, 0.801), (16384, 0.8
 
 def _worse(p, f, M, K):
     """How much larger the squared error is than the fp32 plan's."""
-    e = _squared_error(*p[:4], M, K)
+    e = _squared_error(*p, M, K)
     if _bf16(p):
         k = e
         assert k <= 65536

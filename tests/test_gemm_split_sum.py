@@ -1,4 +1,5 @@
-"""K-split products on the 128 x 64 LDS-direct tiles: each split writes the
+"""K-split products on the 128 x 64 LDS-direct tiles (and, where the planner
+picks it, the 256 x 128 workgroups of the bf16 kernel): each split writes the
 raw product over its K range to a partial plane, and splitk_sum_k adds the
 planes and applies the epilogue.
 
@@ -22,7 +23,7 @@ from gpu_util import announce, down, up
 
 pytestmark = pytest.mark.gpu
 
-TILE_128x64 = 4
+TILE_128x64, TILE_256x128 = 4, 5
 
 
 def _cdiv(a, b):
@@ -40,7 +41,7 @@ def _nan_buffer(native, n):
     return up(native, np.full(n, np.nan, np.float32))
 
 
-def _planes_sum(native, A, B, ranges):
+def _planes_sum(native, A, B, ranges, tile=TILE_128x64):
     """float32 sum over the splits' planes in splitk_sum_k's order."""
     M, N = A.shape[0], B.shape[1]
     planes = []
@@ -48,8 +49,8 @@ def _planes_sum(native, A, B, ranges):
         As, Bs = np.ascontiguousarray(A[:, ks:ke]), np.ascontiguousarray(B[ks:ke])
         dA, dB, dC = up(native, As), up(native, Bs), _nan_buffer(native, M * N)
         native.sgemm_tuned(0, 0, M, N, ke - ks, dA, ke - ks, 0, dB, N, 0, dC, N, 0,
-                           tile=TILE_128x64, splits=1)
-        assert native.last_plan() == [(TILE_128x64, 1, M)], native.last_plan()
+                           tile=tile, splits=1)
+        assert native.last_plan() == [(tile, 1, M)], native.last_plan()
         planes.append(down(native, dC, (M, N)))
     deep = len(planes) >= 8 and M * N // 4 < 65536
     if not deep:
@@ -73,6 +74,7 @@ def _planes_sum(native, A, B, ranges):
     (512, 512, 800, 3),      # the last split shorter (288, 288, 224)
     (256, 2048, 2048, 16),
     (128, 768, 2048, 16),    # 24576 output groups: the planes spread over four waves
+    (2048, 768, 3072, 4),    # a C of 1.5 M elements
 ])
 def test_split_sum_is_the_plane_sum_in_order(native, M, N, K, splits):
     announce(f"split sum {M}x{N}x{K} splits={splits}")
@@ -92,10 +94,11 @@ def test_split_sum_is_the_plane_sum_in_order(native, M, N, K, splits):
     assert np.array_equal(C, want), float(np.max(np.abs(C - want)))
 
 
-@pytest.mark.parametrize("M,N,K", [(1024, 768, 2048), (2048, 768, 3072)])
-def test_split_sum_with_residual_matches_the_plane_sum(native, M, N, K):
-    # silgpu_gemm with bias and residual on the planner's own pick (128 x 64
-    # tiles with a K split for these shapes)
+@pytest.mark.parametrize("M,N,K,tile", [(1024, 768, 2048, TILE_128x64),
+                                        (2048, 768, 3072, TILE_256x128)])
+def test_split_sum_with_residual_matches_the_plane_sum(native, M, N, K, tile):
+    # silgpu_gemm with bias and residual on the planner's own pick (a K split
+    # for these shapes)
     announce(f"split sum residual {M}x{N}x{K}")
     g = rng(17 + M)
     A = g.normal(0, 1, (M, K)).astype(np.float32)
@@ -107,9 +110,9 @@ def test_split_sum_with_residual_matches_the_plane_sum(native, M, N, K):
     native.gemm(0, 0, M, N, K, dA, K, dB, N, dC, N, epi=native.EPI_BIAS, bias=db, bias_len=N,
                 residual=dR, ldr=N)
     plan = native.last_plan()
-    assert len(plan) == 1 and plan[0][0] == TILE_128x64 and plan[0][1] > 1, plan
+    assert len(plan) == 1 and plan[0][0] == tile and plan[0][1] > 1, plan
     C = down(native, dC, (M, N))
-    want = (_planes_sum(native, A, B, _ranges(K, plan[0][1])) + b[None, :]) + R
+    want = (_planes_sum(native, A, B, _ranges(K, plan[0][1]), tile) + b[None, :]) + R
     assert np.array_equal(C, want), float(np.max(np.abs(C - want)))
 
 
