@@ -357,9 +357,10 @@ int silgpu_gemm(const silgpu_gemm_desc *desc);
 int silgpu_gemm_noalloc(const silgpu_gemm_desc *desc);
 
 /* The matrix products the last silgpu_sgemm / silgpu_sgemm_tuned /
- * silgpu_gemm / silgpu_gemm_noalloc call on this thread launched: *n of them
- * (0 for a vector product, which runs the GEMV kernels; 2 when the last
- * rows of C ran as a second product), and for each its tile configuration
+ * silgpu_gemm / silgpu_gemm_noalloc / silgpu_conv2d_f32 call on this thread
+ * launched: *n of them (0 for a vector product, which runs the GEMV kernels, or
+ * a convolution small enough for the direct kernel; 2 when the last rows of C
+ * ran as a second product), and for each its tile configuration
  * (the numbering of silgpu_sgemm_tuned), the K splits it launched and its
  * rows of C.  The arrays hold at least two entries.  No reference
  * counterpart: a diagnostic for tests and tile sweeps. */

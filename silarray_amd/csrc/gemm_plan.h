@@ -99,6 +99,16 @@ inline double plane_bytes(int sp, int64_t M, int64_t N) {
   return sp > 1 ? double(sp) * double(M) * double(N) * 4.0 : 0.0;
 }
 
+// The K splits that fit `room` bytes of scratch, at most sp.
+inline int splits_within(int sp, int64_t M, int64_t N, double room) {
+  if (plane_bytes(sp, M, N) <= room) return sp;
+  const double fit = room / plane_bytes(2, M, N) * 2.0;
+  return fit >= 2.0 ? static_cast<int>(fit) : 1;
+}
+inline bool plan_fits(const plan &p, int64_t M, int64_t N, double room) {
+  return plane_bytes(p.splits, M, N) <= room && plane_bytes(p.tail_splits, p.tail_rows, N) <= room;
+}
+
 inline double plane_sum_time(int sp, int64_t rows, int64_t cols) {
   return 0.8e-6 + double(sp + 1) * double(rows) * double(cols) * 4.0 / 5.0e12 + 0.05e-6 * sp;
 }
@@ -115,17 +125,20 @@ inline double plane_sum_time(int sp, int64_t rows, int64_t cols) {
 // tiles are candidates too.  Nothing runs them (the bf16 kernel is faster), but
 // a product's accuracy is measured against the plan they would have had: an
 // entry point owes no longer K ranges than that.  max_range > 0: the tiles that
-// run, K ranges up to max_range.
+// run, K ranges up to max_range, partial planes within `room`; a time of kNoPlan
+// if there is none.
+constexpr double kNoPlan = 1e30;
 struct fp32_pick {
   plan p;
   double time;
 };
 
 inline fp32_pick fp32_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool dtl_ok,
-                           double max_range) {
+                           double max_range, double room = INFINITY) {
   auto tiles = [&](int bm, int bn) { return cdiv(M, bm) * cdiv(N, bn) * batch; };
-  auto short_enough = [&](const plan &p) {
-    return max_range <= 0.0 || k_range(p, M, K) <= max_range * 1.001;
+  auto allowed = [&](const plan &p) {
+    return max_range <= 0.0 ||
+           (k_range(p, M, K) <= max_range * 1.001 && plan_fits(p, M, N, room));
   };
   // Predicted time of each (tile, K split): every CU runs ceil(WG / 256)
   // workgroups, min(that, occupancy) of them at once; a SIMD holding a
@@ -175,7 +188,7 @@ inline fp32_pick fp32_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool 
     return t > floor_t ? t : floor_t;
   };
   plan best{TILE_128x64, 1};
-  double best_t = 1e30;
+  double best_t = kNoPlan;
   for (const cand &cd : cands) {
     const bool wide = cd.tile == TILE_256x256 || cd.tile == TILE_128x128;
     if (wide && max_range > 0.0) continue;
@@ -183,7 +196,7 @@ inline fp32_pick fp32_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool 
       if (sp > 1 && (batch != 1 || K / sp < 64)) continue;
       // (3- and 6-way splits of the larger tiles won nowhere in the sweeps.)
       if ((sp == 3 || sp == 6) && wide) continue;
-      if (!short_enough(plan{cd.tile, sp})) continue;
+      if (!allowed(plan{cd.tile, sp})) continue;
       if (max_range > 0.0 && double(sp) * max_range > double(K) * 1.001 &&
           plane_bytes(sp, M, N) > kMaxPlaneBytes)
         continue;  // more K splits than accuracy asks for
@@ -217,7 +230,7 @@ inline fp32_pick fp32_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool 
         double t = t_main + round_time(cd, cdiv(mt, cd.bm) * tn * sp, klen) + kLaunch;
         if (sp > 1) t += plane_sum_time(sp, mt, N);
         const plan pl{cd.tile, 1, static_cast<int>(mt), sp};
-        if (t < best_t * 0.97 && short_enough(pl)) {
+        if (t < best_t * 0.97 && allowed(pl)) {
           best_t = t;
           best = pl;
         }
@@ -246,10 +259,10 @@ inline fp32_pick fp32_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool 
     // 51.7 -> 50.8); with shorter groups the two-group tile wins (1024^3
     // 20.9 against 21.5).
     if (sp == 1 && t64 >= 224 && K >= 3072 && K % 128 == 0 &&
-        short_enough(plan{TILE_64x64_K4, 1}))
+        allowed(plan{TILE_64x64_K4, 1}))
       return fp32_pick{plan{TILE_64x64_K4, 1}, 0.0};
     const plan k2{TILE_64x64_K2, static_cast<int>(sp)};
-    if (sp >= 1 && t64 * sp >= 224 && short_enough(k2)) return fp32_pick{k2, 0.0};
+    if (sp >= 1 && t64 * sp >= 224 && allowed(k2)) return fp32_pick{k2, 0.0};
   }
   // Batched products never split K across workgroups; where their 64 x 64
   // tiles fill at most one round of the CUs, the K groups are the only K
@@ -278,7 +291,10 @@ inline fp32_pick fp32_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool 
   return fp32_pick{best, best_t};
 }
 
-inline plan choose_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool dtl_ok, bool vec) {
+// room: bytes of scratch for partial planes (the small-M plans leave theirs to the
+// launch).
+inline plan choose_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool dtl_ok, bool vec,
+                        double room = INFINITY) {
   auto tiles = [&](int bm, int bn) { return cdiv(M, bm) * cdiv(N, bn) * batch; };
   // M <= 32: the small-M kernel (splits chosen at launch), or where it does
   // not apply (batched, A transposed) the 32x128 tile.  Where 32-column
@@ -295,18 +311,26 @@ inline plan choose_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool dtl
   // tiles' K loops: 64x64 measured 25% faster than 128x128 at
   // 48 x 512x512x64 on MI355X.
   if (batch > 1 && K <= 128 && M >= 64 && N >= 64) return plan{TILE_64x64, 1};
-  // The best fp32 plan, and where its tile does not run, the best one that adds
-  // up no longer K ranges on the tiles that do.
-  const fp32_pick ref = fp32_plan(M, N, K, batch, dtl_ok, 0.0);
+  // The best fp32 plan, with the K splits of it that fit, and where it does not run
+  // so, the best one that adds up no longer K ranges on the tiles that do.
+  fp32_pick ref = fp32_plan(M, N, K, batch, dtl_ok, 0.0);
+  const bool wide_ref = ref.p.tile == TILE_256x256 || ref.p.tile == TILE_128x128;
+  const bool fits = plan_fits(ref.p, M, N, room);
+  ref.p.splits = splits_within(ref.p.splits, M, N, room);
+  ref.p.tail_splits = splits_within(ref.p.tail_splits, ref.p.tail_rows, N, room);
   const double range = k_range(ref.p, M, K);
   fp32_pick pick = ref;
   int min_splits = (2 * ref.p.splits + 2) / 3;
-  if (ref.p.tile == TILE_256x256 || ref.p.tile == TILE_128x128) {
-    pick = fp32_plan(M, N, K, batch, dtl_ok, range);
-    // On the bf16 tiles also no fewer than two thirds of the K splits that suit
-    // the tiles that run best.
-    min_splits = (2 * fp32_plan(M, N, K, batch, dtl_ok, INFINITY).p.splits + 2) / 3;
+  if (wide_ref || !fits) {
+    pick = fp32_plan(M, N, K, batch, dtl_ok, range, room);
+    // (5 and 7 splits, say, which no candidate has.)
+    if (pick.time == kNoPlan) pick.p = plan{wide_ref ? TILE_128x64 : ref.p.tile, ref.p.splits};
   }
+  // On the bf16 tiles also no fewer than two thirds of the K splits that suit
+  // the tiles that run best.
+  if (wide_ref)
+    min_splits =
+        (2 * splits_within(fp32_plan(M, N, K, batch, dtl_ok, INFINITY).p.splits, M, N, room) + 2) / 3;
   if (pick.time == 0.0) return pick.p;  // by rule
   // The bf16 kernel's tiles (gemm_split.h), one workgroup per CU: `launch`
   // once, per round of workgroups `fixed` for the first loads and the stores
@@ -332,7 +356,8 @@ inline plan choose_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool dtl
         if (batch != 1 ? sp > 1 || K < 320 : sp > 1 && K / sp < 128) continue;
         if (!exact && (sp == 5 || sp == 16)) continue;
         if (sp < min_splits || (exact && !split_range_ok(double(K) / sp, range))) continue;
-        if (sp > ref.p.splits && plane_bytes(sp, M, N) > kMaxPlaneBytes) continue;
+        if (plane_bytes(sp, M, N) > (sp > ref.p.splits ? std::fmin(room, kMaxPlaneBytes) : room))
+          continue;
         const int64_t wg = tiles(w.bm, w.bn) * sp;
         const double stages = double(cdiv(cdiv(K, sp), w.bk)) + (K % w.bk ? 1.5 : 0.0);
         const double fill = wg < 256 ? double(wg) / 256.0 : 1.0;
@@ -349,6 +374,81 @@ inline plan choose_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool dtl
     if (!wide || exact || split_range_ok(double(K) / best.splits, range)) return best;
   }
   return pick.p;
+}
+
+// A convolution's plan: M output pixels by C_out channels, K = Kd products of which
+// C_in belong to one tap, as a plan of that M x C_out product.  vec: C_in a
+// multiple of 4, operands 16-byte aligned; bf16_ok: sizes that the bf16 kernel's
+// gather takes; room: bytes of scratch for partial planes.
+//
+// The fp32 plan: where nothing is left over, 128 x 64 tiles of the LDS-direct
+// kernel, three workgroups to a CU.  Between one and two tiles per CU (two on some
+// CUs, one on others) the K range is split in two, so the pieces fill three rounds.
+// When the pieces fill whole rounds of all CUs plus a thin last round, the tile rows
+// of that last round run as a second launch split further along K (one piece per CU
+// at most) with its own split sum, instead of a round of a few workgroups at full
+// depth.
+// (Measured: 88.5 -> 85.2 us at 16x28x28x128 -> 256, K = 1152; with K = 576 the
+// halves are too short and the split sum costs more than the balance gains, 48.7 ->
+// 56.6 us at 8x56x56x64 -> 128.)
+inline plan conv_fp32_plan(int64_t M, int64_t C_in, int64_t C_out, int64_t Kd, int64_t cus,
+                           bool vec, double room) {
+  if (!vec || C_in % 16 != 0 || M % 128 != 0 || C_out % 64 != 0)
+    return plan{C_out <= 32 ? TILE_64x64 : TILE_128x64, 1};
+  const int BK = C_in % 32 == 0 ? 32 : 16;
+  const int64_t tiles_n = C_out / 64, tiles_m = M / 128, tiles = tiles_m * tiles_n;
+  const int64_t slots = cus * 3, kt = Kd / BK;
+  const int gs = tiles > cus && 2 * tiles > slots && 4 * (2 * tiles) <= 5 * slots &&
+                         kt % 2 == 0 && Kd >= 1024
+                     ? 2 : 1;
+  const int64_t pieces = tiles * gs, rem = pieces % slots;
+  int64_t tail = 0;
+  int splits = 1;
+  if (pieces > slots && rem > 0 && rem * 4 <= slots) {
+    const int64_t rem_rows = cdiv(rem, tiles_n * gs);
+    tail = rem_rows * 128;
+    for (int64_t sp = 2; sp <= kt; ++sp)
+      if (kt % sp == 0 && rem_rows * tiles_n * sp <= cus) splits = int(sp);
+  }
+  // (The kernel wants whole K tiles in every split: all of them or none.)
+  plan p{TILE_128x64, gs, static_cast<int>(tail), splits};
+  if (plane_bytes(gs, M - tail, C_out) > room) p.splits = 1;
+  if (plane_bytes(splits, tail, C_out) > room) p.tail_splits = 1;
+  return p;
+}
+
+// The bf16 kernel against the fp32 ones, as choose_plan weighs them: its 256 x 128
+// tiles, and K splits, in rounds of the CUs (a K tile costs a sixth more than a
+// product's for the gather) against 92 TFLOP/s on full 128 x 64 tiles and 55 on the
+// register-staged ones, on 3 and 4 workgroups per CU, after 6 us of launch and first
+// loads; of those that sum no longer K ranges, for their error, than the fp32 plan.
+inline plan conv_plan(int64_t M, int64_t C_in, int64_t C_out, int64_t Kd, int64_t cu_count,
+                      bool vec, bool bf16_ok, double room) {
+  plan best = conv_fp32_plan(M, C_in, C_out, Kd, cu_count, vec, room);
+  if (!bf16_ok) return best;
+  const double range = (double(Kd) / best.splits * double(M - best.tail_rows) +
+                        double(Kd) / best.tail_splits * double(best.tail_rows)) / double(M);
+  const bool full_tiles = M % 128 == 0 && C_out % 64 == 0;
+  const double cus = double(cu_count);
+  const double tiles = double(cdiv(M, 128) * cdiv(C_out, 64));
+  const double busy = tiles < cus ? cus / tiles : 1.0;  // idle CUs at full depth
+  double best_t = 0.9 * (6.0e-6 + busy * 2.0 * double(cdiv(M, 128) * 128) *
+                                      double(cdiv(C_out, 64) * 64) * double(Kd) /
+                                      (full_tiles ? 92e12 : 55e12));
+  for (int sp : {1, 2, 3, 4, 6, 8, 12, 16}) {
+    if (sp > 1 && Kd / sp < 128) continue;
+    if (plane_bytes(sp, M, C_out) > room || !split_range_ok(double(Kd) / sp, range)) continue;
+    const double wgs = double(cdiv(M, 256) * cdiv(C_out, 128) * sp);
+    const double fill = wgs < cus ? wgs / cus : 1.0;
+    double t = 5.0e-6 + std::ceil(wgs / cus) * (5.5e-6 + double(cdiv(Kd, 16 * sp)) *
+                                                             (0.92e-6 + 0.28e-6 * fill) * 1.17);
+    if (sp > 1) t += 2.5e-6 + double(sp + 1) * double(M) * double(C_out) * 4.0 / 5.0e12;
+    if (t < best_t) {
+      best_t = t;
+      best = plan{TILE_256x256, sp};
+    }
+  }
+  return best;
 }
 
 }  // namespace

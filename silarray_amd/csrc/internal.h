@@ -149,7 +149,7 @@ constexpr size_t kNoAllocScratchBytes = size_t(32) << 20;  // 32 MiB
 // Whether a launch may use `bytes` of workspace: always, except while the
 // stream is being captured into a graph and the block would have to grow
 // (growing allocates and synchronises, which a capture forbids; the caller
-// then runs a plan without it).
+// then runs a plan that fits).
 bool workspace_available(context *c, size_t bytes);
 // Makes c->workspace hold at least `bytes` (synchronises the stream before
 // replacing a smaller block).

@@ -164,6 +164,7 @@ int set_error(int code, const char *fmt, ...) {
 void clear_error() { g_err[0] = '\0'; }
 
 bool workspace_available(context *c, size_t bytes) {
+  if (bytes == 0) return true;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(c->stream, &st) != hipSuccess || st == hipStreamCaptureStatusNone)
     return true;

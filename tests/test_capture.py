@@ -4,6 +4,9 @@ workspace that a graph uses outlives its growth.  Every replay is compared
 with the eager result, with eager work and synchronisations in between."""
 
 import ctypes as C
+import subprocess
+import sys
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -49,7 +52,9 @@ def test_replays_match_the_eager_result(native):
     def conv():
         native.conv2d(dx, dw, dy, 4, 28, 28, 64, 3, 128)
 
-    gemm(), conv()
+    conv()
+    assert native.last_plan()[0][1] > 1  # a K split, in the workspace by now
+    gemm()
     want_c, want_y = down(native, dC, (M, N)), down(native, dy, (4 * 28 * 28, 128))
     assert native.last_plan()[0][1] > 1  # a K split, in the workspace by now
     graph = Graph(native, lambda: (gemm(), conv()))
@@ -66,27 +71,69 @@ def test_replays_match_the_eager_result(native):
         native.sync()
 
 
-def test_a_split_that_does_not_fit_yet_runs_unsplit(native):
-    announce("capture with a workspace too small")
+def _in_a_new_process(name):
+    """Runs this file's function `name` where no workspace has been allocated yet."""
+    here = Path(__file__).resolve().parent
+    code = (f"import sys; sys.path[:0] = [{str(here)!r}, {str(here.parent)!r}]\n"
+            f"import test_capture as t\nfrom silarray_amd import _native as native\n"
+            f"native.init()\nt.{name}(native)\nprint('done')")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=110)
+    assert r.returncode == 0 and r.stdout.endswith("done\n"), r.stdout + r.stderr
+
+
+def _float64(native, dA, dB, M, N, K):
+    A, B = down(native, dA, (M, K)).astype(np.float64), down(native, dB, (K, N)).astype(np.float64)
+    return A @ B, 1e-5 * np.sqrt(K) * (np.abs(A) @ np.abs(B))
+
+
+def splits_without_room(native):
+    """Products and a convolution whose plans split K, recorded with no workspace:
+    the plans that need none are recorded, and their replays are right."""
     g = rng(4)
-    M, N, K, splits = 2048, 2048, 512, 16
-    need = splits * M * N * 4
-    A, B = g.normal(0, 1, (M, K)).astype(np.float32), g.normal(0, 1, (K, N)).astype(np.float32)
-    dA, dB, dC = up(native, A), up(native, B), empty(native, M * N)
-    native.sgemm_tuned(0, 0, M, N, K, dA, K, 0, dB, N, 0, dC, N, 0, tile=5, splits=1)
-    want = down(native, dC, (M, N))
-    plans = []
+    M, N, K = 700, 600, 2051
+    dA = up(native, g.normal(0, 1, (M, K)).astype(np.float32))
+    dB = up(native, g.normal(0, 1, (K, N)).astype(np.float32))
+    x = g.normal(0, 1, (4, 28, 28, 64)).astype(np.float32)
+    w = g.normal(0, 0.1, (128, 1, 1, 64)).astype(np.float32)
+    w3 = np.zeros((128, 3, 3, 64), np.float32)
+    w3[:, 1, 1] = w[:, 0, 0]  # a 1 x 1 kernel in the middle of a 3 x 3 one
+    dx, dw = up(native, x), up(native, w3)
+    dC, dF, dy = empty(native, M * N), empty(native, M * N), empty(native, 4 * 28 * 28 * 128)
+    plans = {}
+
+    def forced(tile, dst):
+        native.sgemm_tuned(0, 0, M, N, K, dA, K, 0, dB, N, 0, dst, N, 0, tile=tile, splits=8)
 
     def record():
-        native.sgemm_tuned(0, 0, M, N, K, dA, K, 0, dB, N, 0, dC, N, 0, tile=5, splits=splits)
-        plans.extend(native.last_plan())
+        native.gemm(0, 0, M, N, K, dA, K, dB, N, dC, N)
+        plans["gemm"] = native.last_plan()
+        forced(5, dF)
+        plans["forced"] = native.last_plan()
+        native.conv2d(dx, dw, dy, 4, 28, 28, 64, 3, 128)
+        plans["conv"] = native.last_plan()
 
     graph = Graph(native, record)
-    native.call("silgpu_fill_u32", native.vp(dC), 0x7fc00000, M * N)
-    graph.replay()
-    C1 = down(native, dC, (M, N))
-    if plans[0][1] == 1:  # the workspace was smaller than `need`
-        assert np.array_equal(C1, want)
-    else:
-        assert plans[0][1] == splits and need > 0
-        assert np.allclose(C1, want, rtol=0, atol=1e-3)
+    assert all(p[1] == 1 for plan in plans.values() for p in plan), plans
+    assert plans["forced"] == [(5, 1, M)], plans
+    # without K splits the fp32 tiles are ahead of the bf16 kernel's 13 workgroups
+    assert plans["conv"] == [(4, 1, 4 * 28 * 28)], plans
+    want, bar = _float64(native, dA, dB, M, N, K)
+    X, W = x.reshape(-1, 64).astype(np.float64), w.reshape(128, 64).T.astype(np.float64)
+    for rep in range(3):
+        for buf, n in ((dC, M * N), (dF, M * N), (dy, 4 * 28 * 28 * 128)):
+            native.call("silgpu_fill_u32", native.vp(buf), 0x7fc00000, n)
+        graph.replay()
+        for buf in (dC, dF):
+            assert np.all(np.abs(down(native, buf, (M, N)) - want) <= bar)
+        y = down(native, dy, (4 * 28 * 28, 128))
+        assert np.all(np.abs(y - X @ W) <= 1e-5 * 8 * (np.abs(X) @ np.abs(W)))
+        if rep == 0:  # the same calls outside a capture: K splits, and a workspace
+            record()
+            assert plans["gemm"][0][1] > 1 and plans["forced"] == [(5, 8, M)], plans
+            assert plans["conv"][0][1] > 1, plans
+            native.sync()
+
+
+def test_splits_that_do_not_fit_yet_run_without(native):
+    announce("capture without a workspace")
+    _in_a_new_process("splits_without_room")

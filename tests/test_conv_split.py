@@ -21,18 +21,22 @@ def _im2col(x, K):
                            for i in range(K) for j in range(K)], axis=1)
 
 
+TILE_256x128 = 5
+
+
 def _run(native, x, w):
     N, H, W, Ci = x.shape
     Co, K = w.shape[:2]
     dx, dw, dy = up(native, x), up(native, w), empty(native, N * H * W * Co)
     native.conv2d(dx, dw, dy, N, H, W, Ci, K, Co)
+    assert [p[0] for p in native.last_plan()] == [TILE_256x128], native.last_plan()
     return down(native, dy, (N * H * W, Co))
 
 
 @pytest.mark.parametrize("N,H,W,Ci,K,Co", [
     (2, 9, 13, 64, 3, 70), (1, 16, 16, 128, 3, 128), (1, 17, 15, 128, 3, 129),
     (3, 5, 7, 64, 5, 1), (2, 8, 33, 80, 2, 100), (1, 2, 3, 160, 5, 40), (1, 40, 40, 48, 4, 130),
-    (4, 28, 28, 128, 1, 128), (1, 1, 300, 112, 3, 127), (2, 31, 17, 176, 3, 260)])
+    (4, 28, 28, 512, 1, 130), (1, 1, 300, 112, 3, 127), (2, 31, 17, 176, 3, 260)])
 def test_conv_edges(native, N, H, W, Ci, K, Co):
     announce(f"conv split {N}x{H}x{W}x{Ci} k{K} -> {Co}")
     g = rng(N + H + W + Ci + K + Co)

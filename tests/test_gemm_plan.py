@@ -23,8 +23,17 @@ using namespace silgpu;
 int main() {
   long long M, N, K, batch;
   int dtl, vec;
-  while (std::scanf("%lld %lld %lld %lld %d %d", &M, &N, &K, &batch, &dtl, &vec) == 6) {
-    const plan p = choose_plan(M, N, K, batch, dtl, vec);
+  double room;
+  while (std::scanf("%lld %lld %lld %lld %d %d %lf", &M, &N, &K, &batch, &dtl, &vec, &room) == 7) {
+    if (batch < 0) {  // a convolution of K taps of -batch channels
+      const long long Kd = K * -batch;
+      const plan p = conv_plan(M, -batch, N, Kd, 256, vec, vec && batch % 16 == 0, room);
+      const plan f = conv_fp32_plan(M, -batch, N, Kd, 256, vec, room);
+      std::printf("%d %d %d %d  %d %d %d %d\n", p.tile, p.splits, p.tail_rows, p.tail_splits,
+                  f.tile, f.splits, f.tail_rows, f.tail_splits);
+      continue;
+    }
+    const plan p = choose_plan(M, N, K, batch, dtl, vec, room);
     const plan f = fp32_plan(M, N, K, batch, dtl, 0.0).p;
     std::printf("%d %d %d %d  %d %d %d %d\n", p.tile, p.splits, p.tail_rows, p.tail_splits,
                 f.tile, f.splits, f.tail_rows, f.tail_splits);
@@ -41,9 +50,10 @@ def plans(tmp_path_factory):
     subprocess.run([cxx, "-std=c++17", "-O1", f"-I{CSRC}", str(d / "driver.cpp"), "-o",
                     str(d / "driver")], check=True)
 
-    def run(shapes):
-        """[(M, N, K, batch, aligned)] -> [(plan, fp32 plan)]"""
-        text = "".join(f"{M} {N} {K} {b} {int(v and K % 16 == 0)} {int(v)}\n"
+    def run(shapes, room=math.inf):
+        """[(M, N, K, batch, aligned)] -> [(plan, fp32 plan)]; a batch of -c: a
+        convolution, M pixels, K taps of c channels each, N channels out"""
+        text = "".join(f"{M} {N} {K} {b} {int(v and K % 16 == 0)} {int(v)} {room}\n"
                        for M, N, K, b, v in shapes)
         out = subprocess.run([str(d / "driver")], input=text, check=True, capture_output=True,
                              text=True).stdout.split("\n")
@@ -127,3 +137,45 @@ def test_large_products_need_no_workspace_that_they_never_needed(plans):
     for (M, N, K, _, _), (p, f) in zip(shapes, got):
         planes = 4.0 * M * N * p[1] if p[1] > 1 else 0.0
         assert planes <= max(2.0 ** 30, 4.0 * M * N * f[1] if f[1] > 1 else 0.0), (M, N, K, p, f)
+
+
+@pytest.mark.parametrize("room", [0, 5 << 20, 32 << 20])
+def test_plans_within_little_scratch(plans, room):
+    """Where partial planes have to fit (a fixed scratch area, a workspace that may
+    not grow), they do, and no K range is longer, for its error, than those of the
+    fp32 tiles' plan with as many K splits as fit."""
+    rng = random.Random(3)
+    shapes = [(2048, 2048, 32764, 1, False)] + [(*_draw(rng), 1, True) for _ in range(10000)]
+    free, narrow = plans(shapes), plans(shapes, room)
+
+    def planes(p, M, N):
+        return [4 * sp * rows * N for sp, rows in ((p[1], M - p[2]), (p[3], p[2])) if sp > 1]
+
+    changed = 0
+    for (M, N, K, _, _), (p, f), (p0, _) in zip(shapes, narrow, free):
+        assert all(b <= room for b in planes(p, M, N)), (M, N, K, p)
+        if all(b <= room for b in planes(p0, M, N)):
+            assert p == p0 or planes(f, M, N), (M, N, K, p, p0)
+        changed += p != p0
+        fit = [max(1, min(f[1], room // (4 * (M - f[2]) * N))), f[2],
+               max(1, min(f[3], room // (4 * f[2] * N))) if f[2] else 1]
+        assert _worse(p, (f[0], *fit), M, K) <= 1.005, (M, N, K, p, f)
+    assert changed > 100
+
+
+def test_convolutions_add_up_no_longer_ranges(plans):
+    rng = random.Random(4)
+    shapes = [(16 * 56 * 56, 128, 9, -64, True), (4 * 28 * 28, 128, 9, -64, True)]
+    for _ in range(4000):
+        n, hw, k = rng.choice([1, 2, 4, 8, 16]), rng.randint(3, 80), rng.choice([1, 2, 3, 5, 7])
+        shapes.append((n * hw * hw, rng.choice([16, 40, 64, 96, 128, 200, 256, 512]), k * k,
+                       -16 * rng.randint(1, 32), True))
+    for room in (math.inf, 0, 4 << 20):
+        got = plans(shapes, room)
+        assert sum(p[0] == TILE_256x128 for p, _ in got) > 500
+        for (M, N, K, b, _), (p, f) in zip(shapes, got):
+            assert _worse(p, f, M, K * -b) <= 1.005, ((M, N, K, b), p, f)
+            if p[1] > 1:
+                assert 4 * p[1] * (M - p[2]) * N <= room
+            if p[3] > 1:
+                assert 4 * p[3] * p[2] * N <= room
