@@ -33,7 +33,8 @@ struct context {
   // second.  Launches on the one stream run in order, so every call may
   // reuse the whole area.
   void *partials = nullptr;  // kPartialBytes
-  // GEMM split-K workspace: grown to the largest request seen, never shrunk.
+  // GEMM split-K workspace: grown to the largest request seen (to twice its size
+  // where a graph keeps the old block), never shrunk.
   void *workspace = nullptr;
   size_t workspace_bytes = 0;
   bool workspace_captured = false;  // a captured launch uses this block

@@ -176,16 +176,28 @@ bool workspace_available(context *c, size_t bytes) {
 int ensure_workspace(context *c, size_t bytes) {
   if (bytes <= c->workspace_bytes) return SILGPU_OK;
   size_t grow = (bytes + (size_t(64) << 20) - 1) & ~((size_t(64) << 20) - 1);  // 64 MiB steps
+  // A captured graph may replay into the old block, so that is left to the graph, and
+  // the library cannot learn when the graph is gone.  The new block is then at least
+  // twice as large where memory allows: all blocks left behind together stay smaller
+  // than the one in use.
+  const size_t least = grow;
+  if (c->workspace_captured && grow < 2 * c->workspace_bytes) grow = 2 * c->workspace_bytes;
   SILGPU_HIP_CHECK(hipStreamSynchronize(c->stream));
-  // A captured graph may replay into the old block: it is left to the graph.
   if (c->workspace && !c->workspace_captured) SILGPU_HIP_CHECK(hipFree(c->workspace));
   c->workspace_captured = false;
   c->workspace = nullptr;
   c->workspace_bytes = 0;
   hipError_t e = hipMalloc(&c->workspace, grow);
-  if (e != hipSuccess)
+  if (e != hipSuccess && grow > least) {
+    (void)hipGetLastError();
+    grow = least;
+    e = hipMalloc(&c->workspace, grow);
+  }
+  if (e != hipSuccess) {
+    c->workspace = nullptr;
     return set_error(SILGPU_ERR_NOMEM, "GEMM workspace of %zu bytes: %s", grow,
                      hipGetErrorString(e));
+  }
   c->workspace_bytes = grow;
   return SILGPU_OK;
 }

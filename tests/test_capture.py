@@ -137,3 +137,50 @@ def splits_without_room(native):
 def test_splits_that_do_not_fit_yet_run_without(native):
     announce("capture without a workspace")
     _in_a_new_process("splits_without_room")
+
+
+def growth_between_captures(native):
+    """Ten captures, each with the workspace as it is, which then has to grow by
+    64 MiB: every graph keeps its block and replays into it, and all blocks together
+    take no more than four times the largest request (2 GiB of 2.5; one more block of
+    each size would be 3.4 GiB)."""
+    hip = C.CDLL("libamdhip64.so")
+
+    def free():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    g = rng(6)
+    M, N, K = 2048, 2048, 1280
+    dA = up(native, g.normal(0, 1, (M, K)).astype(np.float32))
+    dB = up(native, g.normal(0, 1, (K, N)).astype(np.float32))
+    dC = [empty(native, M * N) for _ in range(11)]
+
+    def product(i, splits):
+        native.sgemm_tuned(0, 0, M, N, K, dA, K, 0, dB, N, 0, dC[i], N, 0, tile=5, splits=splits)
+        if splits == 4:
+            assert native.last_plan() == [(5, 4, M)]
+
+    product(10, 1)  # code objects loaded
+    native.sync()
+    before, graphs = free(), []
+    for i in range(10):
+        product(10, 4 * i + 4)  # 4 (i + 1) planes of 16 MiB
+        graphs.append(Graph(native, lambda: product(i, 4)))
+    native.sync()
+    assert before - free() <= 4 * 640 << 20, (before - free()) >> 20
+    product(10, 4)
+    want = down(native, dC[10], (M, N))
+    for rep in range(3):
+        for i, graph in enumerate(graphs):
+            native.call("silgpu_fill_u32", native.vp(dC[i]), 0x7fc00000, M * N)
+            graph.replay()
+        product(10, 40)
+        for i in range(10):
+            assert np.array_equal(down(native, dC[i], (M, N)), want), (rep, i)
+
+
+def test_workspace_growth_between_captures_is_bounded(native):
+    announce("workspace growth between captures")
+    _in_a_new_process("growth_between_captures")
