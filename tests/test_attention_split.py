@@ -130,6 +130,31 @@ def test_extreme_magnitudes(native, qs, vs):
     assert np.all(np.abs(O - want) <= factor * np.maximum(mag, top * (factor > 1e-3)) + 1e-44)
 
 
+@pytest.mark.parametrize("qs", [1e15, 1e19])
+def test_huge_scores_pick_one_key(native, qs):
+    """Scores around 1e15 (on the bf16 matrix cores) and 1e19 (operands over 2^60:
+    every row redone in fp32).  A score of 64 products errs by at most 64 * 2^-24 of
+    sum |q k|, which is under four times the row's largest score: 2^-16 of that.
+    Where the second score is further off, the row is the value of its first key."""
+    announce(f"attention split: scores about {qs}")
+    g = rng(31)
+    b, Sq, Sk = 200, 128, 576
+    Q = (g.normal(0, 1, (b, Sq, D)) * qs).astype(np.float32)
+    K, V = (g.normal(0, 1, (b, Sk, D)).astype(np.float32) for _ in range(2))
+    O = _run(native, Q, K, V, 0.125)
+    S = Q.astype(np.float64) @ K.astype(np.float64).transpose(0, 2, 1)
+    first = S.argmax(-1)
+    top = np.partition(S, Sk - 2, axis=-1)[..., -2:]
+    largest = np.abs(S).max(-1)
+    mag = np.abs(Q.astype(np.float64)) @ np.abs(K.astype(np.float64)).transpose(0, 2, 1)
+    assert np.all(mag.max(-1) < 4 * largest)
+    clear = top[..., 1] - top[..., 0] > 2.0 ** -16 * largest
+    assert clear.mean() > 0.99
+    want = np.take_along_axis(V, first[..., None], axis=1)
+    assert np.all(np.isfinite(O))
+    assert np.array_equal(O[clear], want[clear])
+
+
 @pytest.mark.parametrize("Sq,Sk", [(128, 576), (97, 530), (130, 31 + 512)])
 def test_values_near_the_bottom_of_the_range(native, Sq, Sk):
     """V elements under 2^-134 have no bf16 part; their averages are not zero.

@@ -198,6 +198,32 @@ def test_rows_of_any_scale_keep_their_accuracy(native, tile):
     assert np.all(np.abs(C - A64 @ B64) <= 1e-5 * np.sqrt(90) * (np.abs(A64) @ np.abs(B64)))
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("tile,M,N,K", [(1, 511, 1027, 333), (5, 700, 1027, 333)])
+def test_batches_of_two_levels(native, tile, M, N, K, ta, tb):
+    """Batched products as the planner sends them here: 2 x 3 of them, the inner
+    three side by side in one row, A's outer stride wider than its product and B the
+    same for both.  In one product every sum is redone on the fp32 matrix cores."""
+    announce(f"bf16 split tile {tile} batched {M}x{N}x{K} ta={ta} tb={tb}")
+    g = rng(M + 2 * ta + tb)
+    ar, ac = (K, M) if ta else (M, K)
+    br, bc = (N, K) if tb else (K, N)
+    A = g.normal(0, 1, (2, ar + 2, 3, ac + 1)).astype(np.float32)
+    B = g.normal(0, 1, (br, 3, bc)).astype(np.float32)
+    A[1, :, 1] *= 1e-34
+    dA, dB = up(native, A), up(native, B)
+    dC = up(native, np.full((2, M, 3, N + 1), 7.0, np.float32))
+    native.gemm(ta, tb, M, N, K, dA, 3 * (ac + 1), dB, 3 * bc, dC, 3 * (N + 1), 2, 3,
+                ((ar + 2) * 3 * (ac + 1), ac + 1), (0, bc), (M * 3 * (N + 1), N + 1))
+    assert native.last_plan() == [(tile, 1, M)], native.last_plan()
+    C = down(native, dC, (2, M, 3, N + 1))
+    assert np.all(C[..., N] == 7.0)
+    for o in range(2):
+        for i in range(3):
+            a, b = A[o, :ar, i, :ac], B[:, i]
+            assert _near_the_bottom(C[o, :, i, :N], a.T if ta else a, b.T if tb else b), (o, i)
+
+
 @pytest.mark.parametrize("K", [96, 768, 4096])
 def test_no_less_accurate_than_the_fp32_instruction(native, K):
     """Against the 64 x 64 tile of the fp32 matrix cores on the same operands."""
