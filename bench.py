@@ -121,6 +121,12 @@ def roofline(bound: str, achieved: float, traffic=None, split=False) -> dict:
             "frac": round(achieved / peak, 4), "traffic": traffic}
 
 
+def on_bf16(plan) -> bool:
+    """Whether the launches that silgpu_gemm_last_plan recorded ran on the bf16
+    matrix cores (tile ids 1 and 5)."""
+    return bool(plan) and all(tile in (1, 5) for tile, *_ in plan)
+
+
 def load_traffic(name: str):
     """HBM bytes per launch measured by rocprofv3 --pmc (FETCH_SIZE +
     WRITE_SIZE, copy-kernel calibrated), committed under profiles/."""
@@ -164,7 +170,8 @@ def bench_sgemm(nat, S, steps, warmup, g, min_warm_s=0.0):
     kern_ms = t.e0.elapsed_ms(t.e1) / steps
     flops = 2.0 * S * S * S
     return {"wall_ms_per_step": wall * 1e3 / steps, "kernel_ms": kern_ms,
-            "tflops_wall": flops / (wall / steps) / 1e12, "tflops_kernel": flops / (kern_ms / 1e3) / 1e12}
+            "tflops_wall": flops / (wall / steps) / 1e12, "tflops_kernel": flops / (kern_ms / 1e3) / 1e12,
+            "split": on_bf16(nat.last_plan())}
 
 
 def bench_gemv(nat, g, reps=200, hot=True):
@@ -218,7 +225,8 @@ def bench_linear_sigmoid(nat, g, reps=50):
     t = Timer(nat)
     ms = t.ms_per_launch(lambda i: nat.sgemm(0, 0, M, N, K, X, K, 0, W, N, 0, Y, N, 0, 1, b, N,
                                              nat.EPI_BIAS_SIGMOID), reps)
-    return {"tflops": 2.0 * M * N * K / (ms / 1e3) / 1e12, "us": ms * 1e3}
+    return {"tflops": 2.0 * M * N * K / (ms / 1e3) / 1e12, "us": ms * 1e3,
+            "split": on_bf16(nat.last_plan())}
 
 
 # The reference's conv2d benchmark layers (bench/micro/bench_nn_ops.cpp:193-195)
@@ -245,7 +253,8 @@ def bench_conv2d(nat, g, reps=50, layers=None):
         out[f"conv2d_{name}_{N}x{Ci}x{H}x{W}_k{K}_co{Co}"] = {
             "tflops": flops / (ms / 1e3) / 1e12, "gbs": nbytes / (ms / 1e3) / 1e9,
             "hbm_bound": flops / nbytes < PEAK_FP32_MFMA_TFLOPS / PEAK_HBM_GBS * 1e3,
-            "us": ms * 1e3, "ref_ms": ref_ms, "traffic_key": f"conv2d_{name}"}
+            "us": ms * 1e3, "ref_ms": ref_ms, "traffic_key": f"conv2d_{name}",
+            "split": on_bf16(nat.last_plan())}
     return out
 
 
@@ -648,7 +657,8 @@ def main():
         log(f"linear_sigmoid {r}")
         secondary["linear_sigmoid_256x4096x4096"] = {
             "value": round(r["tflops"], 2), "unit": "TFLOP/s", "us": round(r["us"], 1),
-            "roofline": roofline("mfma", r["tflops"], load_traffic("linear_sigmoid_256x4096x4096"))}
+            "roofline": roofline("mfma", r["tflops"], load_traffic("linear_sigmoid_256x4096x4096"),
+                                 split=r["split"])}
     conv_layers = {n for n, *_ in CONV_LAYERS if f"conv2d_{n}" in only}
     if want("conv2d") or conv_layers:
         for k, v in bench_conv2d(nat, g, layers=conv_layers or None).items():
@@ -662,7 +672,8 @@ def main():
             else:
                 secondary[k] = {"value": round(v["tflops"], 2), "unit": "TFLOP/s",
                                 "us": round(v["us"], 1), "reference_m1pro_ms": v["ref_ms"],
-                                "roofline": roofline("mfma", v["tflops"], traffic, split=True)}
+                                "roofline": roofline("mfma", v["tflops"], traffic,
+                                                     split=v["split"])}
             # no cpu_baseline: the reference's conv2d has no CPU path
             secondary[k]["cpu_baseline"] = None
             secondary[k]["cpu_baseline_note"] = (
@@ -711,7 +722,7 @@ def main():
             log(f"sgemm {s}^3 {r}")
             secondary[f"sgemm_{s}"] = {"value": round(r["tflops_kernel"], 2), "unit": "TFLOP/s",
                                        "roofline": roofline("mfma", r["tflops_kernel"],
-                                                                split=s > 1024)}
+                                                                split=r["split"])}
 
     if want("graphs"):
         for r in bench_graphs():
@@ -784,7 +795,8 @@ def main():
         line.update({"value": round(r["tflops_wall"], 2), "unit": "TFLOP/s",
                      "ms_per_step": round(r["wall_ms_per_step"], 4),
                      "roofline": roofline("mfma", r["tflops_kernel"],
-                                          load_traffic("sgemm_8192x8192x8192"), split=True)})
+                                          load_traffic("sgemm_8192x8192x8192"),
+                                          split=r["split"])})
     else:
         line.update({"value": None, "unit": "TFLOP/s", "ms_per_step": None, "roofline": None})
     line["cpu_baseline"] = cpu
