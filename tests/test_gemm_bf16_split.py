@@ -168,6 +168,28 @@ def test_one_subnormal_element_anywhere(native, tile, ta, tb):
 
 @pytest.mark.parametrize("tile", [1, 5])
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("few", [True, False])
+def test_sums_that_cancel_beside_sums_that_vanish(native, tile, ta, tb, few):
+    """Sums that are exactly zero because their terms cancel, few and many in a wave's
+    tile, and among them one of elements that have no bf16 part, which is not zero."""
+    announce(f"bf16 split tile {tile} ta={ta} tb={tb}: cancelled sums, few={few}")
+    M, N, K = 300, 150, 330
+    g = rng(K + few)
+    A = g.uniform(0.5, 1, (M, K)).astype(np.float32)
+    B = g.uniform(0.5, 1, (K, N)).astype(np.float32)
+    for m, n in [(0, 0), (129, 37), (299, 149)] if few else \
+            [(m, n) for m in range(0, 300, 9) for n in range(0, 150, 10)]:
+        A[m, 1::2] = -A[m, ::2]
+        B[1::2, n] = B[::2, n]
+    A[70], B[:, 70] = 0.0, 0.0
+    A[70, 11], B[11, 70] = 3e-41, 1000.0
+    C = _run(native, np.ascontiguousarray(A.T) if ta else A,
+             np.ascontiguousarray(B.T) if tb else B, ta, tb, tile)
+    assert _near_the_bottom(C, A, B) and C[70, 70] > 0
+
+
+@pytest.mark.parametrize("tile", [1, 5])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("M,N,K", [(33, 65, 1), (257, 129, 5), (130, 131, 8), (259, 70, 71),
                                    (128, 257, 130)])
 def test_products_redone_whole(native, tile, ta, tb, M, N, K):
