@@ -189,3 +189,21 @@ def test_rows_redone(native, Sq, Sk):
     same = np.ones(O.shape, bool)
     same[::3, :, 63] = same[1::3, :, 2] = False
     assert np.all((np.abs(O - want) <= 2e-5 * mag)[same])
+
+
+@pytest.mark.parametrize("zeros", [1, 3, 9])
+def test_sums_that_cancel_to_zero(native, zeros):
+    """A row of equal weights over a column of V whose values cancel, in few and in
+    many columns: zero to within the rounding of its terms, and next to it a column
+    whose values are too small for bf16 parts, in the same row."""
+    announce(f"attention split: {zeros} columns cancel")
+    g = rng(41 + zeros)
+    b, Sq, Sk = 200, 128, 576
+    Q, K, V = (g.normal(0, 1, (b, s, D)).astype(np.float32) for s in (Sq, Sk, Sk))
+    Q[3, 5] = Q[9, 77] = 0.0
+    V[3, ::2, 7:7 + zeros] = -V[3, 1::2, 7:7 + zeros]
+    V[9, :, 7] = 3e-41
+    O = _run(native, Q, K, V, 0.125)
+    want, mag = _ref(Q, K, V, 0.125)
+    assert np.all(np.abs(O - want) <= 2e-5 * mag + Sk * 2.0 ** -149)
+    assert np.all(O[9, :, 7] > 2.9e-41)
