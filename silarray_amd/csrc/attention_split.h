@@ -24,7 +24,7 @@
 // softmax, split and products one after the other a block took 3.2 and 4.1 us.
 // On the fp32 matrix cores the MFMAs alone took 3.4 us, but there twelve waves
 // fit a CU, so small grids stay there.  MI355X, us, fp32 -> this: heads x
-// queries x keys 24x1000x1000 72.6 -> 52.9, 48x512x512 39.1 -> 30.2,
+// queries x keys 24x1000x1000 70.5 -> 46-47, 48x512x512 39.1 -> 27-30,
 // 16x2048x2048 184 -> 111, 48x2048x2048 510 -> 310, 16x1000x1000 (128
 // workgroups) 54.7 -> 48.7; 24x512x512 27.6 -> 27.6 and 48x300x300 20.2 ->
 // 21.0 stay.  (One after the other, in a run of its own: 76.8 -> 64.9, 40.8 ->
